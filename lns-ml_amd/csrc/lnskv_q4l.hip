@@ -46,7 +46,7 @@ typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kQ4lBlockBytes = LNSKV_Q4L_DEVICE_BYTES;
 constexpr int kQ4lTileVecs = 16;   // vectors per product (A rows)
-constexpr int kQ4lMaxTiles = 4;    // vector tiles per launch (64 vectors)
+constexpr int kQ4lMaxTiles = 4;    // vector tiles of q4l_gemv_acc_kernel (64 vectors)
 constexpr int kQ4lWaves = 4;       // waves per workgroup (split of a range's blocks)
 constexpr int kQ4lTargetWgs = 256; // workgroups wanted per launch: one per CU
 // Buffer resource word 3 for raw dword access (DATA_FORMAT = 32-bit).
@@ -108,10 +108,11 @@ struct Q4lArgs {
   uint32_t* cnt;  // [groups] arrival counts, zero between calls (S > 1)
   uint32_t* err;  // host word set to 1 on a count above S - 1 (a header that was not zero)
   int64_t x_stride, y_stride;
-  int rows, bpr, n_vec, tile0;
+  int rows, bpr, n_vec;
   int groups;     // row groups of 16 q4l_row_tiles(T) rows
   int split;      // S: workgroups per row group
   int bpw;        // blocks per workgroup (the last may hold fewer)
+  int tiles;      // q4l_gemm_acc_kernel: 64-vector tiles (groups = row groups x tiles)
 };
 
 // Workgroup (row group rg, split sp) = blockIdx.x (rg fastest).
@@ -148,7 +149,7 @@ __global__ __launch_bounds__(kQ4lWaves * kWave) void q4l_gemv_acc_kernel(Q4lArgs
   for (int u = 0; u < kPer; ++u) {
     const int idx = tid + u * kQ4lWaves * kWave;
     const int t = idx / (kQ4lTileVecs * RW), v = (idx / RW) % kQ4lTileVecs, r = idx % RW;
-    const int vec = (a.tile0 + t) * kQ4lTileVecs + v;
+    const int vec = t * kQ4lTileVecs + v;
     yv[u] = vec < a.n_vec && row0 + r < a.rows ? a.y[(int64_t)vec * a.y_stride + row0 + r] : 0.0f;
   }
 
@@ -166,7 +167,7 @@ __global__ __launch_bounds__(kQ4lWaves * kWave) void q4l_gemv_acc_kernel(Q4lArgs
   const float* xrow[T];
 #pragma unroll
   for (int t = 0; t < T; ++t) {
-    const int vec = (a.tile0 + t) * kQ4lTileVecs + n;
+    const int vec = t * kQ4lTileVecs + n;
     xrow[t] = a.x + (int64_t)(vec < a.n_vec ? vec : 0) * a.x_stride + 8 * g;
   }
 
@@ -306,9 +307,281 @@ __global__ __launch_bounds__(kQ4lWaves * kWave) void q4l_gemv_acc_kernel(Q4lArgs
   for (int u = 0; u < kPer; ++u) {
     const int idx = tid + u * kQ4lWaves * kWave;
     const int t = idx / (kQ4lTileVecs * RW), v = (idx / RW) % kQ4lTileVecs, r = idx % RW;
-    const int vec = (a.tile0 + t) * kQ4lTileVecs + v;
+    const int vec = t * kQ4lTileVecs + v;
     if (vec >= a.n_vec || row0 + r >= a.rows) continue;
     a.y[(int64_t)vec * a.y_stride + row0 + r] = yv[u] + sum[u];
+  }
+}
+
+// More than 64 vectors (a prompt chunk's o_proj): a workgroup of 8 waves owns
+// 64 vectors x 128 rows; wave w multiplies rows 32 (w % 4) .. with all 64
+// vectors over half w / 4 (128 columns) of every block of its range.  The
+// kernel above re-reads the weights and splits x again for every 64 vectors and
+// every 64 rows; here x is split once per 128 rows, into LDS, and a decoded
+// weight operand serves 64 vectors.
+//   D[vec][row] = sum_k A[vec][k] B[k][row]   (v_mfma_f32_32x32x16_f16)
+// Lane (hl, n) = (lane / 32, lane % 32) holds A of vector n and B of weight
+// row n, k = 8 hl .. + 7, and receives D[vectors 8 (i / 4) + 4 hl + i % 4]
+// [row n].  Of a 32-weight sub-block the lane decodes dwords 2 hl and 2 hl + 1:
+// k step t multiplies the columns 16 hl + 8 t + 0..7, lo and hi parts, four
+// products per sub-block and 32 vectors.
+// A half block's sums stay in the products' accumulators: its weights enter as
+// scale * 2^(m - 5) * 2^k, exact in f16, with one k per row and half block that
+// takes the largest of the four scales to [2^13, 2^14).  The scales of a block
+// are f16(g * 2^(sl - 7)), within 2^15 of each other, so the smallest weight is
+// still a normal number.  (Scales further apart than 2^23, which no disk block
+// has, would lose low bits of weights below 2^-24 of the largest.)  The halves
+// then add up in f32, times 2^-k: 16 multiply-adds for 32 vectors and 128
+// columns instead of 64.
+// x and weights go through LDS a block at a time, both loaded in whole 128-byte
+// lines two blocks ahead.  x in LDS, per half block: [k step s = 2 j + t][hi,
+// lo][hl][vector ^ sw] 16-byte chunks of 8 columns, sw = 2 ((2 s + hl) % 8): 16
+// lanes read 256 contiguous bytes, and the XOR spreads the stores of one
+// vector's chunks over the banks.
+// Bound by issue: a block takes a SIMD's two waves 2048 matrix cycles, ~2450
+// issuing the other vector work (a third of it decoding weights) and, of the
+// LDS, ~3000 (each wave reads the half's 32 KiB of x); what hides one behind
+// another is the order below (without the slices, every LDS read waited for
+// right before its product: 51.7 us).  4096 x 4096: 46.9 us at 512 vectors,
+// 25.0 at 128 (135.3 and 34.5 as launches of 64 vectors); 8192 x 8192 at 600
+// vectors 238 (377).  Waves of 64 rows x a quarter block halve the LDS reads
+// but leave no registers for operands read ahead: 53.7.
+constexpr int kGemmVecs = 64;              // vectors per workgroup
+constexpr int kGemmRows = 128;             // weight rows per workgroup
+constexpr int kGemmWaves = 8;
+constexpr int kGemmOut = kGemmVecs * kGemmRows;
+constexpr int kGemmHalf = 128;             // columns staged at once
+constexpr int kGemmBuf = kGemmVecs * kGemmHalf * 4;  // LDS bytes of one half (hi and lo)
+
+typedef float float16v __attribute__((ext_vector_type(16)));
+typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+
+// weight_codes in the order (w0, w2), (w1, w3), (w4, w6), (w5, w7): the first
+// two dwords belong to columns 0..3, the others to 4..7.
+__device__ __forceinline__ u32x4 weight_codes_split(uint32_t w) {
+  const u32x4 d = weight_codes(w);
+  return u32x4{d.x, d.z, d.y, d.w};
+}
+
+// The hi and lo f16 parts of two x values, both rounded to nearest even (x = hi
+// + lo to 2^-23): x - hi is exact, formed and rounded by one mixed-precision
+// fma of the f16 hi with m1 = -1 (hidden from the compiler as above).
+__device__ __forceinline__ void x_pair_nearest(float a, float b, float m1, uint32_t& hi, uint32_t& lo) {
+  typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+  typedef float float2v __attribute__((ext_vector_type(2)));
+  const half2v h = __builtin_convertvector(float2v{a, b}, half2v);
+  const half2v l = {(_Float16)__builtin_fmaf((float)h[0], m1, a), (_Float16)__builtin_fmaf((float)h[1], m1, b)};
+  hi = __builtin_bit_cast(uint32_t, h);
+  lo = __builtin_bit_cast(uint32_t, l);
+}
+
+// Workgroup barrier after this wave's LDS accesses; unlike __syncthreads() it
+// leaves the loads of the next half in flight.
+__device__ __forceinline__ void gemm_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+__global__ __launch_bounds__(kGemmWaves * kWave) void q4l_gemm_acc_kernel(Q4lArgs a) {
+  constexpr int kChunks = kGemmRows * 9;                                 // 16-byte chunks of a block's weights
+  constexpr int kThreads = kGemmWaves * kWave;
+  constexpr int kLoads = (kChunks + kThreads - 1) / kThreads;
+  __shared__ __attribute__((aligned(16))) uint8_t xs_[4 * kGemmBuf];     // [2 blocks][half]
+  __shared__ __attribute__((aligned(16))) uint8_t ws[kGemmRows * kQ4lBlockBytes];
+  __shared__ int merge;
+  const int tid = (int)threadIdx.x;
+  const int lane = tid & (kWave - 1), w = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int kh = w >> 2;  // the half of every block this wave multiplies (and its threads stage)
+  const int hl = lane >> 5, n = lane & 31;
+  // vector tiles fastest: with blocks dealt to the XCDs in turn, workgroups
+  // that share x (4 bytes a column and vector; the weights are 0.56) share an L2
+  const int vt = (int)blockIdx.x % a.tiles, rest = (int)blockIdx.x / a.tiles;
+  const int rgs = a.groups / a.tiles;
+  const int rg = rest % rgs, sp = rest / rgs;
+  const int vec0 = vt * kGemmVecs, row0 = rg * kGemmRows;
+  const int b0 = sp * a.bpw, nb = min(a.bpr - b0, a.bpw);  // blocks of this split
+
+  // x staging: columns 4c .. 4c + 3 of half kh, vectors sv + 8u; vectors past
+  // n_vec read the last one (never stored).  Loads past the last block re-read
+  // it, unused: a branch around them would make the compiler wait for the
+  // loads of the block before as if none were in flight.
+  const int c = tid & 31, sv = (tid & 255) >> 5;
+  float m1;
+  asm volatile("v_mov_b32 %0, -1.0" : "=v"(m1));
+  float4v xr[8];
+  auto load_x1 = [&](int i, int u) {
+    xr[u] = *reinterpret_cast<const float4v*>(a.x + (int64_t)min(vec0 + sv + 8 * u, a.n_vec - 1) * a.x_stride +
+                                              256 * (b0 + min(i, nb - 1)) + kGemmHalf * kh + 4 * c);
+  };
+  // chunk c / 2: sub-block c / 8, its dword (c / 2) % 4 = 2 hl + t, so k step s
+  const int ss = 2 * (c >> 3) + ((c >> 1) & 1), sh = (c >> 2) & 1;
+  const uint32_t xdst = (uint32_t)(kh * kGemmBuf + ss * 4096 + sh * 1024 + 8 * (c & 1));
+  const uint32_t xsw = 2u * (uint32_t)((2 * ss + sh) & 7);
+  auto stage_x1 = [&](int buf, int u) {
+    uint32_t h0, h1, l0, l1;
+    x_pair_nearest(xr[u][0], xr[u][2], m1, h0, l0);
+    x_pair_nearest(xr[u][1], xr[u][3], m1, h1, l1);
+    uint8_t* dst = xs_ + buf * (2 * kGemmBuf) + xdst + 16u * ((uint32_t)(sv + 8 * u) ^ xsw);
+    *reinterpret_cast<u32x2*>(dst) = u32x2{h0, h1};
+    *reinterpret_cast<u32x2*>(dst + 2048) = u32x2{l0, l1};
+  };
+  // weight staging: chunks tid + 512 u of the tile's rows (rows past the
+  // matrix read its last one)
+  u32x4 wr[kLoads];
+  auto load_w = [&](int i) {
+#pragma unroll
+    for (int u = 0; u < kLoads; ++u) {
+      const int idx = min(tid + kThreads * u, kChunks - 1);
+      wr[u] = *reinterpret_cast<const u32x4*>(
+          a.W + ((int64_t)min(row0 + idx / 9, a.rows - 1) * a.bpr + b0 + min(i, nb - 1)) * kQ4lBlockBytes + 16 * (idx % 9));
+    }
+  };
+  auto stage_w = [&]() {
+#pragma unroll
+    for (int u = 0; u < kLoads; ++u)
+      if (tid + kThreads * u < kChunks) *reinterpret_cast<u32x4*>(ws + 16 * (tid + kThreads * u)) = wr[u];
+  };
+
+  float16v acc[2];
+#pragma unroll
+  for (int q = 0; q < 32; ++q) acc[q >> 4][q & 15] = 0.0f;
+  const uint8_t* wl = ws + (32 * (w & 3) + n) * kQ4lBlockBytes;
+#pragma unroll
+  for (int u = 0; u < 8; ++u) load_x1(0, u);
+  load_w(0);
+#pragma unroll
+  for (int u = 0; u < 8; ++u) {
+    stage_x1(0, u);
+    load_x1(1, u);
+  }
+  stage_w();
+  load_w(1);
+  gemm_barrier();
+  for (int i = 0; i < nb; ++i) {
+    const uint8_t* xb = xs_ + (i & 1) * (2 * kGemmBuf) + kh * kGemmBuf + 1024 * hl;
+    // x operands of sub-block j: [k step][lo, hi][32 vectors]
+    half8 xa[2][2][2][2];
+    auto read_x = [&](int j, half8 (&o)[2][2][2]) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        const uint8_t* x0 = xb + (2 * j + t) * 4096 + 16u * ((uint32_t)n ^ (2u * (uint32_t)((4 * j + 2 * t + hl) & 7)));
+#pragma unroll
+        for (int v = 0; v < 2; ++v) {
+          o[t][0][v] = *reinterpret_cast<const half8*>(x0 + 512 * v + 2048);
+          o[t][1][v] = *reinterpret_cast<const half8*>(x0 + 512 * v);
+        }
+      }
+    };
+    // this lane's weights of the block, then the next block may be stored
+    u32x2 wt[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) wt[j] = *reinterpret_cast<const u32x2*>(wl + 16 + 64 * kh + 16 * j + 8 * hl);
+    const u32x2 scr = *reinterpret_cast<const u32x2*>(wl + 8 * kh);
+    read_x(0, xa[0]);
+    gemm_barrier();
+    // the exponent of the largest |scale| (field e, 2^(e - 15); a subnormal one
+    // counts as e = 1) to 13
+    const uint32_t mag0 = scr[0] & 0x7FFF7FFFu, mag1 = scr[1] & 0x7FFF7FFFu;
+    const uint32_t top = max(max(mag0 & 0xFFFFu, mag0 >> 16), max(mag1 & 0xFFFFu, mag1 >> 16));
+    const int k = 28 - max((int)(top >> 10), 1);
+    auto weights = [&](int j, int t) {
+      const uint32_t sb = scr[j >> 1];
+      const _Float16 s1 =
+          (_Float16)ldexpf((float)__builtin_bit_cast(_Float16, (uint16_t)((j & 1) ? sb >> 16 : sb & 0xFFFFu)), k);
+      return __builtin_bit_cast(half8, weight_codes_split(wt[j][t])) * half8{s1, s1, s1, s1, s1, s1, s1, s1};
+    };
+    float16v d[2];
+#pragma unroll
+    for (int q = 0; q < 32; ++q) d[q >> 4][q & 15] = 0.0f;
+    half8 wa[2][2];  // the weight operands of sub-blocks j and j + 1, [k step]
+    wa[0][0] = weights(0, 0);
+    wa[0][1] = weights(0, 1);
+    // Sub-block j's products, the lo parts first (their roundings are 2^-11 of
+    // the hi parts'); between each two, a slice of the other work: sub-block j +
+    // 1's operands, the next block's x to LDS and the loads of the one after.
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      auto products = [&](int p) {
+#pragma unroll
+        for (int v = 0; v < 2; ++v)
+          d[v] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xa[j & 1][p & 1][p >> 1][v], wa[j & 1][p & 1], d[v], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      __builtin_amdgcn_sched_barrier(0);
+      if (j < 3) read_x(j + 1, xa[(j + 1) & 1]);
+      products(0);
+      stage_x1((i + 1) & 1, 2 * j);  // that buffer was last read before the barrier at this block's start
+      load_x1(i + 2, 2 * j);
+      products(1);
+      if (j < 3) wa[(j + 1) & 1][0] = weights(j + 1, 0);
+      products(2);
+      stage_x1((i + 1) & 1, 2 * j + 1);
+      load_x1(i + 2, 2 * j + 1);
+      products(3);
+      if (j < 3) wa[(j + 1) & 1][1] = weights(j + 1, 1);
+    }
+    stage_w();
+    load_w(i + 2);
+    const float back = ldexpf(1.0f, -k);
+#pragma unroll
+    for (int v = 0; v < 2; ++v)
+#pragma unroll
+      for (int q = 0; q < 16; ++q) acc[v][q] = fmaf(back, d[v][q], acc[v][q]);
+    gemm_barrier();
+  }
+
+  // The two halves of the waves swap: kh = 0 keeps vectors 0..31 of the tile,
+  // kh = 1 vectors 32..63.
+  float* swap = reinterpret_cast<float*>(xs_) + (w & 3) * (16 * kWave) + lane;
+  float16v sum;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    swap[kh * (64 * kWave) + i * kWave] = kh ? acc[0][i] : acc[1][i];
+    sum[i] = kh ? acc[1][i] : acc[0][i];
+  }
+  gemm_barrier();
+#pragma unroll
+  for (int i = 0; i < 16; ++i) sum[i] += swap[(1 - kh) * (64 * kWave) + i * kWave];
+
+  if (a.split > 1) {
+    // as above: the last of the group's splits adds all of them in split order
+    float* part = a.part + (int64_t)(rg * a.tiles + vt) * kGemmOut + tid;
+    const int64_t step = (int64_t)a.groups * kGemmOut;
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+      __hip_atomic_store(part + sp * step + i * kGemmWaves * kWave, sum[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (tid == 0) {
+      uint32_t* cnt = a.cnt + rg * a.tiles + vt;
+      const uint32_t old = __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      const bool all = old == (uint32_t)(a.split - 1);
+      if (old > (uint32_t)(a.split - 1) && a.err)
+        __hip_atomic_store(a.err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      if (all) __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      merge = all;
+    }
+    __syncthreads();
+    if (!merge) return;  // workgroup-uniform
+    for (int s0 = 0; s0 < a.split; ++s0) {
+      float pv[16];
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        pv[i] = __hip_atomic_load(part + s0 * step + i * kGemmWaves * kWave, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+      for (int i = 0; i < 16; ++i) sum[i] = s0 == 0 ? pv[i] : sum[i] + pv[i];
+    }
+  }
+  const int row = row0 + 32 * (w & 3) + n;
+  if (row >= a.rows) return;
+  const int v0 = vec0 + 32 * kh + 4 * hl;  // this lane's vectors: v0 + 8 (i / 4) + i % 4
+  float yv[16];
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const int vec = v0 + 8 * (i >> 2) + (i & 3);
+    yv[i] = vec < a.n_vec ? a.y[(int64_t)vec * a.y_stride + row] : 0.0f;
+  }
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const int vec = v0 + 8 * (i >> 2) + (i & 3);
+    if (vec < a.n_vec) a.y[(int64_t)vec * a.y_stride + row] = yv[i] + sum[i];
   }
 }
 
@@ -330,6 +603,20 @@ void launch_q4l(Q4lArgs a, hipStream_t st) {
   q4l_gemv_acc_kernel<T><<<(unsigned)(a.groups * a.split), kQ4lWaves * kWave, 0, st>>>(a);
 }
 
+// The many-vector kernel's launch.  ws_bytes: what the call's workspace is
+// known to hold (0: none).  Blocks are split over S workgroups while there is
+// a CU without one, each with at least 4 blocks, as far as the workspace holds
+// the partial sums.
+void launch_q4l_gemm(Q4lArgs a, size_t ws_bytes, hipStream_t st) {
+  a.tiles = (a.n_vec + kGemmVecs - 1) / kGemmVecs;
+  a.groups = (a.rows + kGemmRows - 1) / kGemmRows * a.tiles;
+  const size_t fit = ws_bytes > kWsHeaderBytes ? (ws_bytes - kWsHeaderBytes) / (kGemmOut * sizeof(float)) : 0;
+  int S = std::max(1, std::min({kQ4lTargetWgs / a.groups, a.bpr / 4, (int)(fit / (size_t)a.groups)}));
+  a.bpw = (a.bpr + S - 1) / S;
+  a.split = (a.bpr + a.bpw - 1) / a.bpw;
+  q4l_gemm_acc_kernel<<<(unsigned)(a.groups * a.split), kGemmWaves * kWave, 0, st>>>(a);
+}
+
 // Workspace: the arrival counts (LNSKV_WORKSPACE_HEADER_BYTES, zero between
 // calls) and the partial sums of a split launch.  A split needs fewer than
 // kQ4lTargetWgs row groups, so S * groups < 2 kQ4lTargetWgs whatever the rows
@@ -342,8 +629,9 @@ size_t q4l_ws_bytes(int cols, int n_vec) {
   return kWsHeaderBytes + (size_t)2 * kQ4lTargetWgs * (size_t)q4l_wg_outputs(T) * sizeof(float);
 }
 
-// What the launches of one call use: 0 when none of them splits (then the
-// call needs no workspace at all), else at most q4l_ws_bytes(cols, n_vec).
+// The workspace a call asks for: 0 when no launch of its vectors, 64 at a time,
+// splits (then the call needs no workspace at all), else at most
+// q4l_ws_bytes(cols, n_vec).
 size_t q4l_call_ws_bytes(int rows, int cols, int n_vec) {
   const int bpr = cols / 256;
   const int n_tiles = (n_vec + kQ4lTileVecs - 1) / kQ4lTileVecs;
@@ -410,16 +698,17 @@ extern "C" int lnskv_q4l_gemv_accumulate(const void* blocks_dev, const float* x_
   a.rows = rows;
   a.bpr = cols / 256;
   a.n_vec = n_vec;
-  // up to 4 tiles (64 vectors) per launch
-  const int n_tiles = (n_vec + kQ4lTileVecs - 1) / kQ4lTileVecs;
-  for (int t0 = 0; t0 < n_tiles; t0 += kQ4lMaxTiles) {
-    a.tile0 = t0;
-    switch (std::min(n_tiles - t0, kQ4lMaxTiles)) {
-      case 1: launch_q4l<1>(a, st); break;
-      case 2: launch_q4l<2>(a, st); break;
-      case 3: launch_q4l<3>(a, st); break;
-      default: launch_q4l<4>(a, st); break;
-    }
+  // past 64 vectors the gemv kernel would run once per 64: 25.6 us at 65 to 80
+  // vectors and 34.5 at 128 (4096 x 4096), the other kernel 25.0 at both
+  if (n_vec > kQ4lMaxTiles * kQ4lTileVecs) {
+    launch_q4l_gemm(a, need, st);
+    return hip_check("q4l gemm kernel launch");
+  }
+  switch ((n_vec + kQ4lTileVecs - 1) / kQ4lTileVecs) {
+    case 1: launch_q4l<1>(a, st); break;
+    case 2: launch_q4l<2>(a, st); break;
+    case 3: launch_q4l<3>(a, st); break;
+    default: launch_q4l<4>(a, st); break;
   }
   return hip_check("q4l gemv kernel launch");
 }

@@ -67,6 +67,45 @@ def test_q4l_gemv_accumulate(gpu, rows, cols, n_vec, xpad, ypad):
     assert torch.equal(yd2, yd)
 
 
+@pytest.mark.parametrize("rows,cols,n_vec", [
+    (1, 256, 65),        # one row, one block: a tile of 128 rows and one of 64 vectors nearly empty
+    (127, 512, 128),     # one row short of a tile, whole vector tiles
+    (128, 768, 129),     # a whole row tile, one vector in the last tile, an odd count of blocks
+    (129, 2048, 100),    # split: two workgroups of 4 blocks per tile
+    (300, 5120, 191),    # split with a shorter last range
+    (2100, 1280, 257),
+])
+def test_q4l_many_vectors(gpu, rows, cols, n_vec):
+    """More than 64 vectors (tiles of 64 vectors x 128 rows, blocks staged in
+    halves): every vector within the bound of test_q4l_gemv_accumulate at the
+    tiles' edges, padded strides, the padding of y untouched, and the vectors
+    of one call as the calls of up to 64 give them, within both bounds.  Vectors
+    differ in scale by 2^10, the smallest ~2^-4: x in two f16 parts is off by up
+    to 2^-25 however small it is, 5e-7 of a vector of 2^-4."""
+    say("q4l many vectors", rows, cols, n_vec)
+    rng = np.random.default_rng(rows + cols + n_vec)
+    disk = _disk(rng, rows, cols)
+    W = Q4LMatrix(disk, rows, cols, gpu)
+    x = (rng.standard_normal((n_vec, cols + 4)) * np.exp2(rng.uniform(-4, 6, (n_vec, 1)))).astype(np.float32)
+    y0 = rng.standard_normal((n_vec, rows + 3)).astype(np.float32)
+    xd, yd = torch.from_numpy(x).to(gpu), torch.from_numpy(y0).to(gpu)
+    W.gemv_accumulate(xd, yd)
+    few = torch.from_numpy(y0).to(gpu)
+    for v in range(0, n_vec, 64):
+        W.gemv_accumulate(xd[v:v + 64], few[v:v + 64])
+    sync()
+    got = yd.cpu().numpy()
+    dev = W.blocks.cpu().numpy()
+    ref = O.q4l_gemv_f64(dev, x[:, :cols], y0[:, :rows], rows, cols)
+    wabs = np.abs(O.q4l_decode_matrix(dev, rows, cols).astype(np.float64))
+    bound = 2e-6 * (np.abs(x[:, :cols]).astype(np.float64) @ wabs.T + np.abs(y0[:, :rows])) + 1e-30
+    err = np.abs(got[:, :rows] - ref)
+    say("max err / bound", float((err / bound).max()))
+    assert np.all(err <= bound)
+    assert np.all(np.abs(got[:, :rows] - few.cpu().numpy()[:, :rows]) <= 2 * bound)
+    assert np.array_equal(got[:, rows:], y0[:, rows:])
+
+
 def test_q4l_caller_workspace(gpu):
     """A caller's workspace (arrival counts zeroed once) gives the bits of the
     library's buffer, call after call and across shapes that share it (every
