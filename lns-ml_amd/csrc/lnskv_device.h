@@ -59,42 +59,71 @@ constexpr int kDppHalfMirror = 0x141;
 constexpr int kDppMirror = 0x140;
 constexpr int kDppRowShl = 0x100;     // + n: lane i reads lane i+n of its row
 constexpr int kDppRowShr = 0x110;     // + n: lane i reads lane i-n of its row
+constexpr int kDppRowRor = 0x120;     // + n: lane i reads lane (i-n) mod 16 of its row
 constexpr int kDppRowNewBcast = 0x150;  // + n: every lane reads lane n of its row
 
-// Sum over aligned groups of N lanes (N = 1..64, power of two).
+// The pair (x of the lane's own half or 16-lane row, x of the other's), by
+// permlane32_swap / permlane16_swap: an exchange across rows on the VALU (a
+// ds_bpermute goes through LDS, ~100 cycles that a page's score chain waits).
+__device__ __forceinline__ float2 swap_xor32(float x) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(int, x), __builtin_bit_cast(int, x), false, false);
+  return make_float2(__builtin_bit_cast(float, (int)r[0]), __builtin_bit_cast(float, (int)r[1]));
+}
+__device__ __forceinline__ float2 swap_xor16(float x) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(int, x), __builtin_bit_cast(int, x), false, false);
+  return make_float2(__builtin_bit_cast(float, (int)r[0]), __builtin_bit_cast(float, (int)r[1]));
+}
+
+// f over aligned groups of N lanes (N = 1..64, power of two), f commutative
+// and associative up to rounding; every lane of a group gets the same bits.
+template <int N, typename F>
+__device__ __forceinline__ float group_reduce(float x, F f) {
+  if constexpr (N >= 2) x = f(x, dpp_mov<kDppXor1>(x));
+  if constexpr (N >= 4) x = f(x, dpp_mov<kDppXor2>(x));
+  if constexpr (N >= 8) x = f(x, dpp_mov<kDppHalfMirror>(x));
+  if constexpr (N >= 16) x = f(x, dpp_mov<kDppMirror>(x));
+  if constexpr (N >= 32) {
+    const float2 p = swap_xor16(x);
+    x = f(p.x, p.y);
+  }
+  if constexpr (N >= 64) {
+    const float2 p = swap_xor32(x);
+    x = f(p.x, p.y);
+  }
+  return x;
+}
 template <int N>
 __device__ __forceinline__ float group_sum(float x) {
-  if constexpr (N >= 2) x += dpp_mov<kDppXor1>(x);
-  if constexpr (N >= 4) x += dpp_mov<kDppXor2>(x);
-  if constexpr (N >= 8) x += dpp_mov<kDppHalfMirror>(x);
-  if constexpr (N >= 16) x += dpp_mov<kDppMirror>(x);
-  if constexpr (N >= 32) x += __shfl_xor(x, 16);
-  if constexpr (N >= 64) x += __shfl_xor(x, 32);
-  return x;
+  return group_reduce<N>(x, [](float a, float b) { return a + b; });
 }
 template <int N>
 __device__ __forceinline__ float group_max(float x) {
-  if constexpr (N >= 2) x = fmaxf(x, dpp_mov<kDppXor1>(x));
-  if constexpr (N >= 4) x = fmaxf(x, dpp_mov<kDppXor2>(x));
-  if constexpr (N >= 8) x = fmaxf(x, dpp_mov<kDppHalfMirror>(x));
-  if constexpr (N >= 16) x = fmaxf(x, dpp_mov<kDppMirror>(x));
-  if constexpr (N >= 32) x = fmaxf(x, __shfl_xor(x, 16));
-  if constexpr (N >= 64) x = fmaxf(x, __shfl_xor(x, 32));
+  return group_reduce<N>(x, [](float a, float b) { return fmaxf(a, b); });
+}
+// f across lanes that are STRIDE apart (STRIDE a power of two, 4..64):
+// combines the rows of a wave that share a column.
+template <int STRIDE, typename F>
+__device__ __forceinline__ float cross_reduce(float x, F f) {
+  static_assert(STRIDE >= 4 && STRIDE <= 64, "columns span 4..64 lanes");
+  if constexpr (STRIDE <= 8) x = f(x, dpp_mov<kDppRowRor + 8>(x));
+  if constexpr (STRIDE <= 4) x = f(x, dpp_mov<kDppRowRor + 4>(x));  // lanes 8 apart agree by now
+  if constexpr (STRIDE <= 16) {
+    const float2 p = swap_xor16(x);
+    x = f(p.x, p.y);
+  }
+  if constexpr (STRIDE <= 32) {
+    const float2 p = swap_xor32(x);
+    x = f(p.x, p.y);
+  }
   return x;
 }
-// Sum / max across lanes that are STRIDE apart (STRIDE power of two): combines
-// the rows of a wave that share a column.
 template <int STRIDE>
 __device__ __forceinline__ float cross_sum(float x) {
-#pragma unroll
-  for (int o = STRIDE; o < kWave; o <<= 1) x += __shfl_xor(x, o);
-  return x;
+  return cross_reduce<STRIDE>(x, [](float a, float b) { return a + b; });
 }
 template <int STRIDE>
 __device__ __forceinline__ float cross_max(float x) {
-#pragma unroll
-  for (int o = STRIDE; o < kWave; o <<= 1) x = fmaxf(x, __shfl_xor(x, o));
-  return x;
+  return cross_reduce<STRIDE>(x, [](float a, float b) { return fmaxf(a, b); });
 }
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
