@@ -95,6 +95,10 @@ struct PfLanes {
 template <int RPW>
 __device__ __forceinline__ void pf_issue(const PrefillArgs& a, const PfLanes& pl, uint32_t page_bytes,
                                          uint32_t kvh_off, lds_u8* slot, uint32_t ph0, uint32_t ph1, int w) {
+  // uniform: with w in a vector register each DMA's resource counted as per
+  // lane and was issued in a loop over its values (32 seqs x 128 tokens, 32/8
+  // heads of 128, f16: 668 us, now 657; 256-wide Q8A heads 882, now 843)
+  w = __builtin_amdgcn_readfirstlane(w);
 #pragma unroll
   for (int t = 0; t < RPW; ++t) {
     const int r = (w >> 2) * RPW + t;  // wave-uniform
@@ -132,6 +136,7 @@ template <int NH>
 __device__ __forceinline__ void pf_issue_q8(const PrefillArgs& a, uint32_t rs, uint32_t kvh, lds_u8* slot,
                                             uint32_t ph0, uint32_t ph1, int w) {
   typedef __attribute__((address_space(3))) void lds_void;
+  w = __builtin_amdgcn_readfirstlane(w);  // as above
   const int lane = (int)(threadIdx.x & (kWave - 1));
   const uint32_t page_bytes = kPage * rs;
 #pragma unroll
