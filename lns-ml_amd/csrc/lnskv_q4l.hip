@@ -363,13 +363,14 @@ __device__ __forceinline__ u32x4 weight_codes_split(uint32_t w) {
   return u32x4{d.x, d.z, d.y, d.w};
 }
 
-// The hi and lo f16 parts of two x values, both rounded to nearest even (x = hi
-// + lo to 2^-23): x - hi is exact, formed and rounded by one mixed-precision
-// fma of the f16 hi with m1 = -1 (hidden from the compiler as above).
-__device__ __forceinline__ void x_pair_nearest(float a, float b, float m1, uint32_t& hi, uint32_t& lo) {
+// The hi and lo f16 parts of two x values: hi rounded toward zero (so that a
+// finite x past 65504 keeps a finite hi and the rest in lo, to 131008), lo to
+// nearest even (x = hi + lo to 2^-22): x - hi is exact, formed and rounded by
+// one mixed-precision fma of the f16 hi with m1 = -1 (hidden from the compiler
+// as above).
+__device__ __forceinline__ void x_pair_split(float a, float b, float m1, uint32_t& hi, uint32_t& lo) {
   typedef _Float16 half2v __attribute__((ext_vector_type(2)));
-  typedef float float2v __attribute__((ext_vector_type(2)));
-  const half2v h = __builtin_convertvector(float2v{a, b}, half2v);
+  const auto h = __builtin_amdgcn_cvt_pkrtz(a, b);
   const half2v l = {(_Float16)__builtin_fmaf((float)h[0], m1, a), (_Float16)__builtin_fmaf((float)h[1], m1, b)};
   hi = __builtin_bit_cast(uint32_t, h);
   lo = __builtin_bit_cast(uint32_t, l);
@@ -416,8 +417,8 @@ __global__ __launch_bounds__(kGemmWaves * kWave) void q4l_gemm_acc_kernel(Q4lArg
   const uint32_t xsw = 2u * (uint32_t)((2 * ss + sh) & 7);
   auto stage_x1 = [&](int buf, int u) {
     uint32_t h0, h1, l0, l1;
-    x_pair_nearest(xr[u][0], xr[u][2], m1, h0, l0);
-    x_pair_nearest(xr[u][1], xr[u][3], m1, h1, l1);
+    x_pair_split(xr[u][0], xr[u][2], m1, h0, l0);
+    x_pair_split(xr[u][1], xr[u][3], m1, h1, l1);
     uint8_t* dst = xs_ + buf * (2 * kGemmBuf) + xdst + 16u * ((uint32_t)(sv + 8 * u) ^ xsw);
     *reinterpret_cast<u32x2*>(dst) = u32x2{h0, h1};
     *reinterpret_cast<u32x2*>(dst + 2048) = u32x2{l0, l1};

@@ -106,6 +106,26 @@ def test_q4l_many_vectors(gpu, rows, cols, n_vec):
     assert np.array_equal(got[:, rows:], y0[:, rows:])
 
 
+@pytest.mark.parametrize("n_vec", [64, 65])
+def test_q4l_x_past_f16_range(gpu, n_vec):
+    """|x| above 65504, which a nearest-even hi part would make infinite: hi is
+    65504 and lo the rest, both exact here (multiples of 32), so the bound of
+    test_q4l_gemv_accumulate holds on both sides of the kernels' dividing line."""
+    say("q4l large x", n_vec)
+    rng = np.random.default_rng(n_vec)
+    rows, cols = 130, 512
+    disk = _disk(rng, rows, cols)
+    W = Q4LMatrix(disk, rows, cols, gpu)
+    x = rng.choice(np.array([65536.0, -65536.0, 98304.0, -131008.0, 1.0], np.float32), (n_vec, cols))
+    yd = torch.zeros((n_vec, rows), device=gpu)
+    W.gemv_accumulate(torch.from_numpy(x).to(gpu), yd)
+    sync()
+    dev = W.blocks.cpu().numpy()
+    ref = O.q4l_gemv_f64(dev, x, np.zeros((n_vec, rows), np.float32), rows, cols)
+    wabs = np.abs(O.q4l_decode_matrix(dev, rows, cols).astype(np.float64))
+    assert np.all(np.abs(yd.cpu().numpy() - ref) <= 2e-6 * (np.abs(x).astype(np.float64) @ wabs.T) + 1e-30)
+
+
 def test_q4l_caller_workspace(gpu):
     """A caller's workspace (arrival counts zeroed once) gives the bits of the
     library's buffer, call after call and across shapes that share it (every
