@@ -20,10 +20,10 @@
 //
 // Bound by VALU issue from about four query heads per kv head on (one head: by
 // HBM).  The sums and maxima across rows stay on the VALU (DPP and permlane
-// swaps) and a page rescales the accumulators only when a running max moves by
-// more than kValuSlack: 48 sequences, 8 heads per kv head, head_dim 64 take
-// 74.8 us on f16 pages and 151 on Q8A (82.7 and 206 with ds_bpermute exchanges
-// and a rescale per page).
+// swaps) and a page of f16 or Q8A rescales the accumulators only when a running
+// max moves by more than kValuSlack: 48 sequences, 8 heads per kv head, head_dim
+// 64, contexts 256 to 4096 take 81.9 us on f16 pages and 159 on Q8A (89.2 and 206
+// with ds_bpermute exchanges and a rescale per page).
 #include "lnskv_device.h"
 
 namespace lnskv {
@@ -43,7 +43,11 @@ __device__ __forceinline__ float elem(const uint4& raw, int e) {
   }
 }
 
-constexpr float kValuSlack = 8.0f;  // log2 units the running max may lag
+// log2 units the running max may lag.  Weights then reach 2^slack, which f16
+// values times any count of tokens leave far from overflow; values of f32 and
+// Q8A pages may themselves lie near the top of f32, so there the max is exact.
+template <int DT>
+constexpr float kValuSlack = DT == LNSKV_DTYPE_F16 ? 8.0f : 0.0f;
 
 template <int DT, int D, int REP>
 struct Geo {
@@ -125,16 +129,19 @@ __device__ __forceinline__ void consume_page(WaveState<DT, D, REP>& st, const Pa
   // head's page max exceeds it by more than the slack (rare after the first
   // pages; weights stay below 2^kValuSlack otherwise).
   float mx[REP];
-  bool need = false;
+  // f32 pages: every page rescales; with no slack some head's max moves on most
+  // pages and the test cost more than it saved (48 sequences, 8 heads per kv
+  // head, head_dim 64: 91.2 us; 87.5 with every page rescaling)
+  bool need = DT == LNSKV_DTYPE_F32;
 #pragma unroll
   for (int h = 0; h < REP; ++h) {
     float x = s[0][h];
 #pragma unroll
     for (int j = 1; j < G::NLOAD; ++j) x = fmaxf(x, s[j][h]);
     mx[h] = cross_max<G::LPR>(x);  // the same in every lane
-    need |= mx[h] > st.m[h] + kValuSlack;
+    need |= mx[h] > st.m[h] + kValuSlack<DT>;
   }
-  if (__builtin_amdgcn_ballot_w64(need)) {  // wave-uniform
+  if (DT == LNSKV_DTYPE_F32 || __builtin_amdgcn_ballot_w64(need)) {  // wave-uniform
 #pragma unroll
     for (int h = 0; h < REP; ++h) {
       const float m_new = fmaxf(st.m[h], mx[h]);

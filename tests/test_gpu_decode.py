@@ -196,6 +196,32 @@ def test_large_query_values_keep_precision(gpu):
     assert rel_err(out, ref).max() < TOL[DTYPE_F16]
 
 
+@pytest.mark.parametrize("d,rep", [(64, 8), (128, 1), (256, 2)])
+def test_large_values_do_not_overflow(gpu, d, rep):
+    """f32 pages, one late token with V near the top of f32 and a score up to 7
+    (log2 units) above the earlier ones: its weight relative to the running
+    bound stays at most 1, so the sum stays finite."""
+    say("large v", d, rep)
+    L = 900
+    pk, tables, kv_len, q = _case(gpu, DTYPE_F32, d, rep, 2, (L,), seed=5)
+    k, v = np.zeros((2, pk.k.numel()), np.float32).reshape(2, *pk.k.shape)
+    late = L - 3
+    page = tables[0, late // 16]
+    k[page, late % 16, :, 0] = 1.0
+    v[page, late % 16] = 1.0e37
+    q[:] = 0.0
+    q[..., 0] = np.linspace(0.0, 7.0 * np.log(2.0), q.shape[1], dtype=np.float32)
+    pk.k.copy_(torch.from_numpy(k))
+    pk.v.copy_(torch.from_numpy(v))
+    hp, _ = host_pages(pk)
+    ref = O.decode_f64(hp, q, tables, kv_len, None, 1.0)
+    for split in (0, 512, 1024):
+        out = pk.decode(dev_f32(q, gpu), dev_i32(tables, gpu), dev_i32(kv_len, gpu), n_heads=2 * rep, max_kv_len=L,
+                        scale=1.0, split=split)
+        sync()
+        assert rel_err(out, ref).max() < TOL[DTYPE_F32]
+
+
 def test_reference_single_sequence_call_c1_shape(gpu):
     """lnskv_attention_paged: the reference's encode_attention_paged_q8a call
     (append token `pos`, attend [p_start, pos], scale rsqrt(d)), here on the
