@@ -330,9 +330,12 @@ int lnskv_q4l_prepare(const void* disk_blocks, size_t disk_bytes, int32_t rows, 
  * workspace_dev/ws_bytes: 16-byte aligned device scratch of at least
  * lnskv_q4l_workspace_size(cols, n_vec) bytes (0 when cols < 2048: no
  * workspace is read), or NULL/0 to use a buffer the library keeps per device.
- * A call none of whose launches splits its rows' blocks (enough row groups to
- * fill the GPU, e.g. rows >= 8192 for up to 16 vectors) reads no workspace and
- * may pass NULL without the library buffer being grown, under capture too.
+ * A call that does not split its rows' blocks (enough work to fill the GPU,
+ * e.g. rows >= 8192 for up to 16 vectors, 4096 rows for 512) reads no workspace
+ * and may pass NULL without the library buffer being grown, under capture too.
+ * A smaller workspace, or a library buffer that cannot grow under capture, is
+ * refused, except that above 64 vectors one that holds what calls of 64 would
+ * use is taken: the rows' blocks are then split, and summed, in fewer parts.
  * It holds the partial sums of a launch that splits each row's blocks over
  * several workgroups, after LNSKV_WORKSPACE_HEADER_BYTES of arrival counts
  * that must be zero before the first use (hipMemset once); every call leaves

@@ -473,10 +473,13 @@ int launch_prefill_mfma(const PrefillArgs& a, int rep, int head_dim, int n_tiles
 
 int hip_check(const char* what);
 // A device buffer the library keeps per device: 0 the decode workspace, 1
-// RoPE'd q/k rows, 2 the Q4L GEMV's x operands.  Growing it allocates a new
+// RoPE'd q/k rows, 2 the Q4L GEMV's partial sums.  Growing it allocates a new
 // buffer and keeps the old one until lnskv_workspace_release (no device
 // synchronization inside a call); during stream capture it fails with
 // LNSKV_ERR_WORKSPACE instead.  Calls that share one must not overlap in time.
 int library_buffer(int which, size_t need, void** out, hipStream_t stream);
+// The same, except that a buffer that cannot grow serves as it is if it holds
+// `least` bytes; *have (may be null) is what it holds.
+int library_buffer(int which, size_t need, size_t least, void** out, size_t* have, hipStream_t stream);
 
 }  // namespace lnskv

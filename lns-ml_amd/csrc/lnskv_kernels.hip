@@ -557,28 +557,39 @@ int grow_locked(int dev, int which, size_t need) {
 }  // namespace
 
 int library_buffer(int which, size_t need, void** out, hipStream_t stream) {
+  return library_buffer(which, need, need, out, nullptr, stream);
+}
+
+int library_buffer(int which, size_t need, size_t least, void** out, size_t* have, hipStream_t stream) {
   if (which < 0 || which >= kLibraryBuffers) return fail(LNSKV_ERR_INVALID, "library buffer %d", which);
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) return fail(LNSKV_ERR_HIP, "hipGetDevice failed");
   std::lock_guard<std::mutex> lock(g_ws_mutex);
   const size_t slot = (size_t)dev * kLibraryBuffers + (size_t)which;
-  if (g_ws.size() <= slot || g_ws[slot].bytes < need) {
+  const size_t held = g_ws.size() > slot ? g_ws[slot].bytes : 0;
+  if (held < need) {
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(stream, &cs) != hipSuccess) {
       (void)hipGetLastError();
       return fail(LNSKV_ERR_HIP, "hipStreamIsCapturing failed");
     }
-    if (cs != hipStreamCaptureStatusNone)
-      return fail(LNSKV_ERR_WORKSPACE,
-                  "the library %s holds %zu bytes, this call needs %zu, and the stream is being captured: "
-                  "pass a workspace or call lnskv_workspace_reserve before capturing",
-                  kBufferName[which], g_ws.size() > slot ? g_ws[slot].bytes : (size_t)0, need);
-    if (int rc = grow_locked(dev, which, need)) return rc;
-    // a decode or Q4L workspace starts with its counts at zero
-    if ((which == 0 || which == 2) && hipMemsetAsync(g_ws[slot].ptr, 0, kWsHeaderBytes, stream) != hipSuccess)
+    const bool serves = held > 0 && held >= least;  // as it is
+    if (cs != hipStreamCaptureStatusNone) {
+      if (!serves)
+        return fail(LNSKV_ERR_WORKSPACE,
+                    "the library %s holds %zu bytes, this call needs %zu, and the stream is being captured: "
+                    "pass a workspace or call lnskv_workspace_reserve before capturing",
+                    kBufferName[which], held, need);
+    } else if (int rc = grow_locked(dev, which, need)) {
+      if (!serves) return rc;
+      clear_error();
+    } else if ((which == 0 || which == 2) && hipMemsetAsync(g_ws[slot].ptr, 0, kWsHeaderBytes, stream) != hipSuccess) {
+      // a decode or Q4L workspace starts with its counts at zero
       return fail(LNSKV_ERR_HIP, "hipMemsetAsync of the workspace header failed");
+    }
   }
   *out = g_ws[slot].ptr;
+  if (have) *have = g_ws[slot].bytes;
   return LNSKV_OK;
 }
 

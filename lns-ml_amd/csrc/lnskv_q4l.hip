@@ -350,6 +350,7 @@ constexpr int kGemmVecs = 64;              // vectors per workgroup
 constexpr int kGemmRows = 128;             // weight rows per workgroup
 constexpr int kGemmWaves = 8;
 constexpr int kGemmOut = kGemmVecs * kGemmRows;
+constexpr size_t kGemmPartBytes = kGemmOut * sizeof(float);  // partial sums of one workgroup
 constexpr int kGemmHalf = 128;             // columns staged at once
 constexpr int kGemmBuf = kGemmVecs * kGemmHalf * 4;  // LDS bytes of one half (hi and lo)
 
@@ -604,18 +605,22 @@ void launch_q4l(Q4lArgs a, hipStream_t st) {
   q4l_gemv_acc_kernel<T><<<(unsigned)(a.groups * a.split), kQ4lWaves * kWave, 0, st>>>(a);
 }
 
-// The many-vector kernel's launch.  ws_bytes: what the call's workspace is
-// known to hold (0: none).  Blocks are split over S workgroups while there is
-// a CU without one, each with at least 4 blocks, as far as the workspace holds
-// the partial sums.
-void launch_q4l_gemm(Q4lArgs a, size_t ws_bytes, hipStream_t st) {
-  a.tiles = (a.n_vec + kGemmVecs - 1) / kGemmVecs;
-  a.groups = (a.rows + kGemmRows - 1) / kGemmRows * a.tiles;
-  const size_t fit = ws_bytes > kWsHeaderBytes ? (ws_bytes - kWsHeaderBytes) / (kGemmOut * sizeof(float)) : 0;
-  int S = std::max(1, std::min({kQ4lTargetWgs / a.groups, a.bpr / 4, (int)(fit / (size_t)a.groups)}));
-  a.bpw = (a.bpr + S - 1) / S;
-  a.split = (a.bpr + a.bpw - 1) / a.bpw;
-  q4l_gemm_acc_kernel<<<(unsigned)(a.groups * a.split), kGemmWaves * kWave, 0, st>>>(a);
+// The many-vector kernel's plan: blocks are split over S workgroups while there
+// is a CU without one (its LDS holds one workgroup), each with at least 4 blocks
+// (four take 13.5 us at 1024 x 1024, four and a merge 18.2 at 1024 x 4096), as
+// far as a workspace of ws_bytes holds the partial sums.  Us with this split |
+// within the partial sums of 64-vector launches (half the workgroups or fewer) |
+// as such launches: 65 vectors, 4096 x 4096 20.7 | 25.2 | 24.3, 8192 x 8192
+// 47.9 | 71.6 | 56.4, 16 x 4096 17.2 | 36.6 | 20.3; 129 vectors, 4096 x 14336
+// 70.2 | 118 | 96.9.
+void q4l_gemm_plan(Q4lArgs* a, size_t ws_bytes) {
+  a->tiles = (a->n_vec + kGemmVecs - 1) / kGemmVecs;
+  a->groups = (a->rows + kGemmRows - 1) / kGemmRows * a->tiles;
+  const size_t fit = ws_bytes > kWsHeaderBytes ? (ws_bytes - kWsHeaderBytes) / kGemmPartBytes : 0;
+  const int by_shape = std::min(kQ4lTargetWgs / a->groups, a->bpr / 4);
+  const int S = std::max(1, (int)std::min((size_t)by_shape, fit / (size_t)a->groups));
+  a->bpw = (a->bpr + S - 1) / S;
+  a->split = (a->bpr + a->bpw - 1) / a->bpw;
 }
 
 // Workspace: the arrival counts (LNSKV_WORKSPACE_HEADER_BYTES, zero between
@@ -630,10 +635,10 @@ size_t q4l_ws_bytes(int cols, int n_vec) {
   return kWsHeaderBytes + (size_t)2 * kQ4lTargetWgs * (size_t)q4l_wg_outputs(T) * sizeof(float);
 }
 
-// The workspace a call asks for: 0 when no launch of its vectors, 64 at a time,
-// splits (then the call needs no workspace at all), else at most
+// What launches of the gemv kernel, 64 vectors at a time, use: 0 when none of
+// them splits (then they need no workspace at all), else at most
 // q4l_ws_bytes(cols, n_vec).
-size_t q4l_call_ws_bytes(int rows, int cols, int n_vec) {
+size_t q4l_gemv_ws_bytes(int rows, int cols, int n_vec) {
   const int bpr = cols / 256;
   const int n_tiles = (n_vec + kQ4lTileVecs - 1) / kQ4lTileVecs;
   size_t most = 0;
@@ -677,32 +682,46 @@ extern "C" int lnskv_q4l_gemv_accumulate(const void* blocks_dev, const float* x_
       (reinterpret_cast<uintptr_t>(blocks_dev) & 15) != 0)
     return fail(LNSKV_ERR_INVALID, "x and the blocks must be 16-byte aligned and x_stride a multiple of 4");
   const hipStream_t st = (hipStream_t)stream;
-  const size_t need = q4l_call_ws_bytes(rows, cols, n_vec);
-  if (need > 0) {
-    if (ws == nullptr) {
-      if (int rc = library_buffer(2, need, &ws, st)) return rc;
-    } else if (ws_bytes < need) {
-      return fail(LNSKV_ERR_WORKSPACE, "workspace of %zu bytes, %zu needed", ws_bytes, need);
-    } else if ((reinterpret_cast<uintptr_t>(ws) & 15) != 0) {
-      return fail(LNSKV_ERR_WORKSPACE, "workspace must be 16-byte aligned");
-    }
-  }
   Q4lArgs a{};
   a.W = static_cast<const uint8_t*>(blocks_dev);
   a.x = x_dev;
   a.y = y_dev;
-  a.cnt = need > 0 ? static_cast<uint32_t*>(ws) : nullptr;
-  a.part = need > 0 ? reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + kWsHeaderBytes) : nullptr;
-  a.err = need > 0 ? ws_error_word(stream, true) : nullptr;
   a.x_stride = x_stride;
   a.y_stride = y_stride;
   a.rows = rows;
   a.bpr = cols / 256;
   a.n_vec = n_vec;
-  // past 64 vectors the gemv kernel would run once per 64: 25.6 us at 65 to 80
-  // vectors and 34.5 at 128 (4096 x 4096), the other kernel 25.0 at both
-  if (n_vec > kQ4lMaxTiles * kQ4lTileVecs) {
-    launch_q4l_gemm(a, need, st);
+  const bool many = n_vec > kQ4lMaxTiles * kQ4lTileVecs;
+  // need: what the launch uses.  The many-vector kernel also takes a workspace
+  // below the size query's answer, or a library buffer that cannot grow under
+  // capture, that holds what gemv launches would use, and then splits less.
+  size_t need = q4l_gemv_ws_bytes(rows, cols, n_vec), least = need;
+  if (many) {
+    q4l_gemm_plan(&a, SIZE_MAX);
+    need = a.split > 1 ? kWsHeaderBytes + (size_t)a.split * (size_t)a.groups * kGemmPartBytes : 0;
+    least = std::min(least, need);
+  }
+  if (need > 0) {
+    size_t have = ws_bytes;
+    if (ws == nullptr) {
+      if (int rc = library_buffer(2, need, least, &ws, &have, st)) return rc;
+    } else if (ws_bytes < least) {
+      return fail(LNSKV_ERR_WORKSPACE, "workspace of %zu bytes, %zu needed", ws_bytes, need);
+    } else if ((reinterpret_cast<uintptr_t>(ws) & 15) != 0) {
+      return fail(LNSKV_ERR_WORKSPACE, "workspace must be 16-byte aligned");
+    }
+    if (have < need) q4l_gemm_plan(&a, least);
+    a.cnt = static_cast<uint32_t*>(ws);
+    a.part = reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + kWsHeaderBytes);
+    a.err = ws_error_word(stream, true);
+  }
+  // past 64 vectors the gemv kernel would run once per 64.  Over 418 shapes of
+  // 16 to 50000 rows, 256 to 14336 columns and 65 to 640 vectors the other kernel
+  // took less time at every one: nearest (0.99) for a second round of a few
+  // workgroups (16385 x 14336 at 65 vectors, 251.8 us against 254.2), 20.7
+  // against 24.3 at 4096 x 4096 and 65, 48.1 against 139.5 at 512
+  if (many) {
+    q4l_gemm_acc_kernel<<<(unsigned)(a.groups * a.split), kGemmWaves * kWave, 0, st>>>(a);
     return hip_check("q4l gemm kernel launch");
   }
   switch ((n_vec + kQ4lTileVecs - 1) / kQ4lTileVecs) {

@@ -4,7 +4,7 @@ sum_c |W[r][c] x[c]| + |y_in| (f32 sums of exact f16 x f16 products: ~cols/32
 f32 roundings of the sub-block partial sums, x split into two f16 parts
 rounded toward zero, to 2^-20; measured at most 1.8e-7 at 4096 columns.
 Dropping the lo part of x would give ~2^-11).  Shapes cover one vector, odd counts, row counts that
-are not multiples of 16, padded strides, more than 64 vectors (two passes),
+are not multiples of 16, padded strides, more than 64 vectors (the other kernel),
 the Llama-3-8B o_proj shape at batch 32 and wider rows whose waves take two
 blocks each (the next block's weights arriving during the products); every
 call gives the same bits, and the padding of y is not written."""
@@ -37,7 +37,7 @@ def _disk(rng, rows, cols):
     (4096, 4096, 32, 0, 0),
     (2048, 8192, 3, 0, 0),    # split launch, two blocks per wave (one vector tile)
     (4096, 8192, 24, 4, 0),   # split launch, two blocks per wave (two vector tiles)
-    (512, 4096, 70, 0, 3),    # two split launches (4 tiles, then 1) sharing the arrival counts
+    (512, 4096, 70, 0, 3),    # more than 64 vectors, split over four workgroups per tile
 ])
 def test_q4l_gemv_accumulate(gpu, rows, cols, n_vec, xpad, ypad):
     say("q4l gemv", rows, cols, n_vec, xpad, ypad)
@@ -67,21 +67,42 @@ def test_q4l_gemv_accumulate(gpu, rows, cols, n_vec, xpad, ypad):
     assert torch.equal(yd2, yd)
 
 
-@pytest.mark.parametrize("rows,cols,n_vec", [
-    (1, 256, 65),        # one row, one block: a tile of 128 rows and one of 64 vectors nearly empty
-    (127, 512, 128),     # one row short of a tile, whole vector tiles
-    (128, 768, 129),     # a whole row tile, one vector in the last tile, an odd count of blocks
-    (129, 2048, 100),    # split: two workgroups of 4 blocks per tile
-    (300, 5120, 191),    # split with a shorter last range
-    (2100, 1280, 257),
+PART_BYTES = 64 * 128 * 4  # a workgroup's partial sums in a split launch of more than 64 vectors
+
+
+def _split_parts(W, x, y, gpu):
+    """y += W x with a caller's workspace whose partial area holds a NaN
+    pattern: the PART_BYTES pieces that the call wrote (workgroups per tile
+    times tiles; 0 when it did not split).  Its arrival counts are left zero."""
+    from lnskv import _lib
+    ws = torch.full((_lib.WORKSPACE_HEADER_BYTES + 256 * PART_BYTES,), 0xFF, dtype=torch.uint8, device=gpu)
+    ws[:_lib.WORKSPACE_HEADER_BYTES] = 0
+    assert W.workspace_size(x.shape[0]) <= ws.numel()
+    W.gemv_accumulate(x, y, ws)
+    sync()
+    assert int(ws[:_lib.WORKSPACE_HEADER_BYTES].count_nonzero()) == 0
+    return int((ws[_lib.WORKSPACE_HEADER_BYTES:].view(-1, PART_BYTES) != 0xFF).any(1).sum())
+
+
+@pytest.mark.parametrize("rows,cols,n_vec,split", [
+    (1, 256, 65, 1),        # one row, one block: a tile of 128 rows and one of 64 vectors nearly empty
+    (127, 512, 128, 1),     # one row short of a tile, whole vector tiles
+    (128, 768, 129, 1),     # a whole row tile, one vector in the last tile, an odd count of blocks
+    (129, 2048, 100, 2),    # two workgroups of 4 blocks per tile
+    (300, 5120, 191, 5),    # five workgroups of 4 blocks per tile
+    (300, 5632, 191, 5),    # the last of five with 2 blocks, the others with 5
+    (16, 4096, 65, 4),      # one row group: the blocks limit the split
+    (2100, 1280, 257, 1),
+    (4096, 4096, 100, 4),   # 64 tiles: one workgroup per CU limits the split
 ])
-def test_q4l_many_vectors(gpu, rows, cols, n_vec):
-    """More than 64 vectors (tiles of 64 vectors x 128 rows, blocks staged in
-    halves): every vector within the bound of test_q4l_gemv_accumulate at the
-    tiles' edges, padded strides, the padding of y untouched, and the vectors
-    of one call as the calls of up to 64 give them, within both bounds.  Vectors
-    differ in scale by 2^10, the smallest ~2^-4: x in two f16 parts is off by up
-    to 2^-25 however small it is, 5e-7 of a vector of 2^-4."""
+def test_q4l_many_vectors(gpu, rows, cols, n_vec, split):
+    """More than 64 vectors (tiles of 64 vectors x 128 rows, a row's blocks
+    split over `split` workgroups): every vector within the bound of
+    test_q4l_gemv_accumulate at the tiles' edges, padded strides, the padding of
+    y untouched, the vectors of one call as the calls of up to 64 give them,
+    within both bounds, and a caller's workspace the bits of the library's
+    buffer.  Vectors differ in scale by 2^10, the smallest ~2^-4: x in two f16
+    parts is off by up to 2^-25 however small it is, 5e-7 of a vector of 2^-4."""
     say("q4l many vectors", rows, cols, n_vec)
     rng = np.random.default_rng(rows + cols + n_vec)
     disk = _disk(rng, rows, cols)
@@ -104,6 +125,53 @@ def test_q4l_many_vectors(gpu, rows, cols, n_vec):
     assert np.all(err <= bound)
     assert np.all(np.abs(got[:, :rows] - few.cpu().numpy()[:, :rows]) <= 2 * bound)
     assert np.array_equal(got[:, rows:], y0[:, rows:])
+    own = torch.from_numpy(y0).to(gpu)
+    tiles = ((rows + 127) // 128) * ((n_vec + 63) // 64)
+    assert _split_parts(W, xd, own, gpu) == (split * tiles if split > 1 else 0)
+    assert torch.equal(own, yd)
+
+
+def test_q4l_many_vectors_small_workspace(gpu):
+    """A workspace below lnskv_q4l_workspace_size that holds what launches of 64
+    vectors at a time would use (4096 x 4096: 4 workgroups for each of 64 row
+    groups of 64 rows, 16 KiB each) is taken, with fewer workgroups per tile;
+    so is a library buffer of that size under capture.  One below is refused
+    and leaves y as it was."""
+    from lnskv import _lib
+    from lnskv._lib import check, lib
+    say("q4l many vectors, small workspace")
+    rng = np.random.default_rng(31)
+    rows, cols, n_vec = 4096, 4096, 100
+    W = Q4LMatrix(_disk(rng, rows, cols), rows, cols, gpu)
+    x = torch.from_numpy(rng.standard_normal((n_vec, cols)).astype(np.float32)).to(gpu)
+    y0 = torch.from_numpy(rng.standard_normal((n_vec, rows)).astype(np.float32)).to(gpu)
+    least = _lib.WORKSPACE_HEADER_BYTES + 4 * 64 * 16384
+    assert least < W.workspace_size(n_vec)
+    ws = torch.zeros(least, dtype=torch.uint8, device=gpu)
+    want = y0.clone()
+    W.gemv_accumulate(x, want, ws)
+    y = y0.clone()
+    with pytest.raises(RuntimeError, match="workspace"):
+        W.gemv_accumulate(x, y, ws[:least - 16])
+    sync()
+    assert torch.equal(y, y0)
+    ref = y0.double() + x.double() @ torch.from_numpy(
+        O.q4l_decode_matrix(W.blocks.cpu().numpy(), rows, cols)).to(gpu).double().t().contiguous()
+    assert float((want.double() - ref).norm() / ref.norm()) < 6e-7
+    check(lib().lnskv_workspace_release())
+    check(lib().lnskv_workspace_reserve(0, 0, least))
+    sync()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        W.gemv_accumulate(x, y)
+    for rep in range(3):
+        y.copy_(y0)
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, want), rep
+    del g
+    torch.cuda.synchronize()
+    check(lib().lnskv_workspace_release())
 
 
 @pytest.mark.parametrize("n_vec", [64, 65])
@@ -134,7 +202,7 @@ def test_q4l_caller_workspace(gpu):
     from lnskv import _lib
     say("q4l caller workspace")
     rng = np.random.default_rng(11)
-    shapes = [(4096, 4096, 32), (1000, 2048, 5), (4096, 4096, 64)]
+    shapes = [(4096, 4096, 32), (1000, 2048, 5), (4096, 4096, 64), (300, 5632, 191), (4096, 4096, 100)]
     mats = {}
     need = 0
     for rows, cols, n_vec in shapes:
@@ -165,16 +233,17 @@ def test_q4l_caller_workspace(gpu):
     assert int(y.count_nonzero()) == 0
 
 
-def test_q4l_graph_replay_library_buffer(gpu):
+@pytest.mark.parametrize("n_vec", [32, 100])
+def test_q4l_graph_replay_library_buffer(gpu, n_vec):
     """lnskv_workspace_reserve grows the library's Q4L buffer (its arrival
     counts zeroed) before a capture; the captured y = y0; y += W x (a split
-    launch, 4096 x 4096 with 32 vectors) then replays with unrelated eager
+    launch, 4096 x 4096, of either kernel) then replays with unrelated eager
     work between the replays, each replay equal to the eager call bit for
     bit, so the counts are back at zero after every replay."""
     from lnskv._lib import check, lib
     say("q4l graph replay")
     rng = np.random.default_rng(21)
-    rows, cols, n_vec = 4096, 4096, 32
+    rows, cols = 4096, 4096
     W = Q4LMatrix(_disk(rng, rows, cols), rows, cols, gpu)
     check(lib().lnskv_workspace_reserve(0, 0, W.workspace_size(n_vec)))
     x = torch.from_numpy(rng.standard_normal((n_vec, cols)).astype(np.float32)).to(gpu)

@@ -70,9 +70,10 @@ def test_decode_poisoned_header_is_reported(gpu, monkeypatch):
         _drain_report()
 
 
-def test_q4l_poisoned_header_is_reported(gpu):
-    say("q4l split launch, poisoned workspace header")
-    rows, cols, n_vec = 4096, 4096, 32
+@pytest.mark.parametrize("n_vec", [32, 100])
+def test_q4l_poisoned_header_is_reported(gpu, n_vec):
+    say("q4l split launch, poisoned workspace header", n_vec)
+    rows, cols = 4096, 4096
     rng = np.random.default_rng(9)
     n = rows * (cols // 256)
     disk = rng.integers(0, 256, (n, O.Q4L_DISK_BYTES), dtype=np.uint8)
@@ -98,12 +99,14 @@ def test_q4l_poisoned_header_is_reported(gpu):
         _drain_report()
 
 
-def test_q4l_unsplit_call_needs_no_workspace(gpu):
-    """8192 rows with up to 16 vectors fill the GPU without splitting a row's
-    blocks: such a call reads no workspace, so a NULL workspace works under
-    graph capture without growing the library buffer."""
-    say("q4l unsplit call under capture, NULL workspace")
-    rows, cols, n_vec = 8192, 2048, 8
+@pytest.mark.parametrize("rows,n_vec", [(8192, 8), (2048, 1024)])
+def test_q4l_unsplit_call_needs_no_workspace(gpu, rows, n_vec):
+    """8192 rows with up to 16 vectors, or 256 tiles of 128 rows and 64 vectors,
+    fill the GPU without splitting a row's blocks: such a call reads no
+    workspace, so a NULL workspace works under graph capture without growing
+    the library buffer, and so does one that holds nothing."""
+    say("q4l unsplit call under capture, NULL workspace", rows, n_vec)
+    cols = 2048
     rng = np.random.default_rng(13)
     n = rows * (cols // 256)
     disk = rng.integers(0, 256, (n, O.Q4L_DISK_BYTES), dtype=np.uint8)
@@ -128,3 +131,7 @@ def test_q4l_unsplit_call_needs_no_workspace(gpu):
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(y, eager)
+    y.copy_(y0)
+    W.gemv_accumulate(x, y, torch.full((16,), POISON, dtype=torch.uint8, device=gpu))
+    sync()
+    assert torch.equal(y, eager)
