@@ -19,11 +19,11 @@
 // and rows are summed once at the end.
 //
 // Bound by VALU issue from about four query heads per kv head on (one head: by
-// HBM).  The sums and maxima across rows stay on the VALU (DPP and permlane
-// swaps) and a page of f16 or Q8A rescales the accumulators only when a running
-// max moves by more than kValuSlack: 48 sequences, 8 heads per kv head, head_dim
-// 64, contexts 256 to 4096 take 81.9 us on f16 pages and 159 on Q8A (89.2 and 206
-// with ds_bpermute exchanges and a rescale per page).
+// HBM).  Where its exchanges across rows run (VALU swaps or LDS) and whether a
+// page tests that a running max moved before it rescales is chosen per page
+// type and head count (Geo).  48 sequences, 8 heads per kv head, head_dim 64,
+// contexts 256 to 4096: 81.8 us on f16 pages and 152.8 on Q8A (89.0 and 206 with
+// every exchange across rows through LDS; f16 83.2 without the test).
 #include "lnskv_device.h"
 
 namespace lnskv {
@@ -43,9 +43,10 @@ __device__ __forceinline__ float elem(const uint4& raw, int e) {
   }
 }
 
-// log2 units the running max may lag.  Weights then reach 2^slack, which f16
-// values times any count of tokens leave far from overflow; values of f32 and
-// Q8A pages may themselves lie near the top of f32, so there the max is exact.
+// log2 units the running max may lag where a page tests (Geo::kTest).  Weights
+// then reach 2^slack, which f16 values times any count of tokens leave far from
+// overflow; values of f32 and Q8A pages may themselves lie near the top of f32,
+// so there the max is exact.
 template <int DT>
 constexpr float kValuSlack = DT == LNSKV_DTYPE_F16 ? 8.0f : 0.0f;
 
@@ -57,6 +58,19 @@ struct Geo {
   static constexpr int RPL = kWave / LPR;    // rows per load
   static constexpr int NLOAD = kPage / RPL;  // loads per page
   static_assert(LPR >= 4 && LPR <= 64, "row must span 4..64 lanes");
+  // A page raises the running maxima and rescales the accumulators only if some
+  // head's page max exceeds them by more than the slack (wave-uniform test)
+  // instead of always.  Us, tested | always, head_dim 64, 48 sequences: f16 8
+  // heads 81.8 | 83.2, 4 heads 45.9 | 43.8 (two registers more: three waves a
+  // SIMD, not four), 1 and 2 within 1%.  Without slack some head's max moves on
+  // most pages: Q8A 8 heads 159 | 153, 4 59.0 | 57.5, 2 33.2 | 33.5; f32 8 heads
+  // 91.2 | 87.5.
+  static constexpr bool kTest = DT == LNSKV_DTYPE_F16 ? REP != 4 : DT == LNSKV_DTYPE_Q8A && REP <= 2;
+  // The accumulators are summed over the wave's rows at the end through LDS on
+  // f16 pages with up to 4 heads, where four or more waves a SIMD hide the wait
+  // (4 heads 41.6 us, 43.8 by swaps); by swaps otherwise (Q8A, 4 heads: 57.5, 62
+  // through LDS).
+  static constexpr bool kSumLds = DT == LNSKV_DTYPE_F16 && REP <= 4;
 };
 
 // Loads one page (K and V chunks of this lane, plus Q8A per-token scales).
@@ -125,23 +139,17 @@ __device__ __forceinline__ void consume_page(WaveState<DT, D, REP>& st, const Pa
       for (int h = 0; h < REP; ++h) s[j][h] = -INFINITY;
     }
   }
-  // The running max is raised, and the accumulators rescaled, only when some
-  // head's page max exceeds it by more than the slack (rare after the first
-  // pages; weights stay below 2^kValuSlack otherwise).
   float mx[REP];
-  // f32 pages: every page rescales; with no slack some head's max moves on most
-  // pages and the test cost more than it saved (48 sequences, 8 heads per kv
-  // head, head_dim 64: 91.2 us; 87.5 with every page rescaling)
-  bool need = DT == LNSKV_DTYPE_F32;
+  bool need = !G::kTest;
 #pragma unroll
   for (int h = 0; h < REP; ++h) {
     float x = s[0][h];
 #pragma unroll
     for (int j = 1; j < G::NLOAD; ++j) x = fmaxf(x, s[j][h]);
     mx[h] = cross_max<G::LPR>(x);  // the same in every lane
-    need |= mx[h] > st.m[h] + kValuSlack<DT>;
+    if constexpr (G::kTest) need |= mx[h] > st.m[h] + kValuSlack<DT>;
   }
-  if (DT == LNSKV_DTYPE_F32 || __builtin_amdgcn_ballot_w64(need)) {  // wave-uniform
+  if (!G::kTest || __builtin_amdgcn_ballot_w64(need)) {  // wave-uniform
 #pragma unroll
     for (int h = 0; h < REP; ++h) {
       const float m_new = fmaxf(st.m[h], mx[h]);
@@ -354,9 +362,9 @@ __global__ __launch_bounds__(kBlock) void decode_valu_kernel(DecodeArgs a) {
   // Rows -> wave totals (every row holds the same m).
 #pragma unroll
   for (int h = 0; h < REP; ++h) {
-    st.l[h] = cross_sum<G::LPR>(st.l[h]);
+    st.l[h] = cross_sum<G::LPR, G::kSumLds>(st.l[h]);
 #pragma unroll
-    for (int e = 0; e < G::EPL; ++e) st.acc[h][e] = cross_sum<G::LPR>(st.acc[h][e]);
+    for (int e = 0; e < G::EPL; ++e) st.acc[h][e] = cross_sum<G::LPR, G::kSumLds>(st.acc[h][e]);
   }
   if (r == 0) {
 #pragma unroll

@@ -62,9 +62,10 @@ constexpr int kDppRowShr = 0x110;     // + n: lane i reads lane i-n of its row
 constexpr int kDppRowRor = 0x120;     // + n: lane i reads lane (i-n) mod 16 of its row
 constexpr int kDppRowNewBcast = 0x150;  // + n: every lane reads lane n of its row
 
-// The pair (x of the lane's own half or 16-lane row, x of the other's), by
-// permlane32_swap / permlane16_swap: an exchange across rows on the VALU (a
-// ds_bpermute goes through LDS, ~100 cycles that a page's score chain waits).
+// The pair (x of the lower, x of the upper) of the two halves, or of the two
+// 16-lane rows of a half, that hold the lane, the same pair in both: an exchange
+// across rows on the VALU by permlane32_swap / permlane16_swap (a ds_bpermute
+// goes through LDS, ~100 cycles that a page's score chain waits).
 __device__ __forceinline__ float2 swap_xor32(float x) {
   const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(int, x), __builtin_bit_cast(int, x), false, false);
   return make_float2(__builtin_bit_cast(float, (int)r[0]), __builtin_bit_cast(float, (int)r[1]));
@@ -101,25 +102,31 @@ __device__ __forceinline__ float group_max(float x) {
   return group_reduce<N>(x, [](float a, float b) { return fmaxf(a, b); });
 }
 // f across lanes that are STRIDE apart (STRIDE a power of two, 4..64):
-// combines the rows of a wave that share a column.
-template <int STRIDE, typename F>
+// combines the rows of a wave that share a column.  LDS: by ds_bpermute, which
+// costs a wait but two VALU instructions instead of four; the bits are the same.
+template <int STRIDE, bool LDS = false, typename F>
 __device__ __forceinline__ float cross_reduce(float x, F f) {
   static_assert(STRIDE >= 4 && STRIDE <= 64, "columns span 4..64 lanes");
-  if constexpr (STRIDE <= 8) x = f(x, dpp_mov<kDppRowRor + 8>(x));
-  if constexpr (STRIDE <= 4) x = f(x, dpp_mov<kDppRowRor + 4>(x));  // lanes 8 apart agree by now
-  if constexpr (STRIDE <= 16) {
-    const float2 p = swap_xor16(x);
-    x = f(p.x, p.y);
-  }
-  if constexpr (STRIDE <= 32) {
-    const float2 p = swap_xor32(x);
-    x = f(p.x, p.y);
+  if constexpr (LDS) {
+#pragma unroll
+    for (int o = STRIDE; o < kWave; o <<= 1) x = f(x, __shfl_xor(x, o));
+  } else {
+    if constexpr (STRIDE <= 8) x = f(x, dpp_mov<kDppRowRor + 8>(x));
+    if constexpr (STRIDE <= 4) x = f(x, dpp_mov<kDppRowRor + 4>(x));  // lanes 8 apart agree by now
+    if constexpr (STRIDE <= 16) {
+      const float2 p = swap_xor16(x);
+      x = f(p.x, p.y);
+    }
+    if constexpr (STRIDE <= 32) {
+      const float2 p = swap_xor32(x);
+      x = f(p.x, p.y);
+    }
   }
   return x;
 }
-template <int STRIDE>
+template <int STRIDE, bool LDS = false>
 __device__ __forceinline__ float cross_sum(float x) {
-  return cross_reduce<STRIDE>(x, [](float a, float b) { return a + b; });
+  return cross_reduce<STRIDE, LDS>(x, [](float a, float b) { return a + b; });
 }
 template <int STRIDE>
 __device__ __forceinline__ float cross_max(float x) {
