@@ -66,6 +66,11 @@ struct Geo {
   // most pages: Q8A 8 heads 159 | 153, 4 59.0 | 57.5, 2 33.2 | 33.5; f32 8 heads
   // 91.2 | 87.5.
   static constexpr bool kTest = DT == LNSKV_DTYPE_F16 ? REP != 4 : DT == LNSKV_DTYPE_Q8A && REP <= 2;
+  // A token's score is summed across 16-lane rows (rows of 512 and 1024 bytes)
+  // through LDS with 8 heads, where VALU issue is the bound: f32, head_dim 256,
+  // 184 us (203 by swaps), head_dim 128 375 (379); by swaps otherwise (f32,
+  // head_dim 256, 2 heads: 113, 117 through LDS).
+  static constexpr bool kScoreLds = REP == 8;
   // The accumulators are summed over the wave's rows at the end through LDS on
   // f16 pages with up to 4 heads, where four or more waves a SIMD hide the wait
   // (4 heads 41.6 us, 43.8 by swaps); by swaps otherwise (Q8A, 4 heads: 57.5, 62
@@ -125,7 +130,7 @@ __device__ __forceinline__ void consume_page(WaveState<DT, D, REP>& st, const Pa
       float part = 0.0f;
 #pragma unroll
       for (int e = 0; e < G::EPL; ++e) part = fmaf(elem<DT>(pr.k[j], e), st.q[h][e], part);
-      s[j][h] = group_sum<G::LPR>(part);
+      s[j][h] = group_sum<G::LPR, G::kScoreLds>(part);
       if constexpr (DT == LNSKV_DTYPE_Q8A) s[j][h] *= pr.ks[j];
     }
   }

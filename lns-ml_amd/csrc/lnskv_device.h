@@ -77,33 +77,39 @@ __device__ __forceinline__ float2 swap_xor16(float x) {
 
 // f over aligned groups of N lanes (N = 1..64, power of two), f commutative
 // and associative up to rounding; every lane of a group gets the same bits.
-template <int N, typename F>
+// LDS: the exchanges across rows by ds_bpermute, one VALU instruction each beside
+// the wait instead of three or four; the bits are the same.
+template <int N, bool LDS = false, typename F>
 __device__ __forceinline__ float group_reduce(float x, F f) {
   if constexpr (N >= 2) x = f(x, dpp_mov<kDppXor1>(x));
   if constexpr (N >= 4) x = f(x, dpp_mov<kDppXor2>(x));
   if constexpr (N >= 8) x = f(x, dpp_mov<kDppHalfMirror>(x));
   if constexpr (N >= 16) x = f(x, dpp_mov<kDppMirror>(x));
-  if constexpr (N >= 32) {
-    const float2 p = swap_xor16(x);
-    x = f(p.x, p.y);
-  }
-  if constexpr (N >= 64) {
-    const float2 p = swap_xor32(x);
-    x = f(p.x, p.y);
+  if constexpr (LDS) {
+    if constexpr (N >= 32) x = f(x, __shfl_xor(x, 16));
+    if constexpr (N >= 64) x = f(x, __shfl_xor(x, 32));
+  } else {
+    if constexpr (N >= 32) {
+      const float2 p = swap_xor16(x);
+      x = f(p.x, p.y);
+    }
+    if constexpr (N >= 64) {
+      const float2 p = swap_xor32(x);
+      x = f(p.x, p.y);
+    }
   }
   return x;
 }
-template <int N>
+template <int N, bool LDS = false>
 __device__ __forceinline__ float group_sum(float x) {
-  return group_reduce<N>(x, [](float a, float b) { return a + b; });
+  return group_reduce<N, LDS>(x, [](float a, float b) { return a + b; });
 }
 template <int N>
 __device__ __forceinline__ float group_max(float x) {
   return group_reduce<N>(x, [](float a, float b) { return fmaxf(a, b); });
 }
 // f across lanes that are STRIDE apart (STRIDE a power of two, 4..64):
-// combines the rows of a wave that share a column.  LDS: by ds_bpermute, which
-// costs a wait but two VALU instructions instead of four; the bits are the same.
+// combines the rows of a wave that share a column.  LDS as above.
 template <int STRIDE, bool LDS = false, typename F>
 __device__ __forceinline__ float cross_reduce(float x, F f) {
   static_assert(STRIDE >= 4 && STRIDE <= 64, "columns span 4..64 lanes");
