@@ -196,30 +196,67 @@ def test_large_query_values_keep_precision(gpu):
     assert rel_err(out, ref).max() < TOL[DTYPE_F16]
 
 
+@pytest.mark.parametrize("dtype", [DTYPE_F32, DTYPE_Q8A])
 @pytest.mark.parametrize("d,rep", [(64, 8), (128, 1), (256, 2)])
-def test_large_values_do_not_overflow(gpu, d, rep):
-    """f32 pages, one late token with V near the top of f32 and a score up to 7
-    (log2 units) above the earlier ones: its weight relative to the running
-    bound stays at most 1, so the sum stays finite."""
-    say("large v", d, rep)
+def test_large_values_do_not_overflow(gpu, dtype, d, rep):
+    """f32 and Q8A pages, one late token with V near the top of f32 and a score
+    up to 7 (log2 units) above the earlier ones: its weight relative to the
+    running bound stays at most 1, so the sum stays finite (a weight of 2^7
+    would make it 1.3e39).  Q8A: codes of 127 with the scale 1 / 127 times those
+    values; a split of the caller's keeps 128- and 256-wide heads on the generic
+    kernel."""
+    say("large v", DTYPE_NAMES[dtype], d, rep)
     L = 900
-    pk, tables, kv_len, q = _case(gpu, DTYPE_F32, d, rep, 2, (L,), seed=5)
-    k, v = np.zeros((2, pk.k.numel()), np.float32).reshape(2, *pk.k.shape)
+    pk, tables, kv_len, q = _case(gpu, dtype, d, rep, 2, (L,), seed=5)
+    q8 = dtype == DTYPE_Q8A
+    k, v = np.zeros((2, pk.k.numel()), np.int8 if q8 else np.float32).reshape(2, *pk.k.shape)
     late = L - 3
     page = tables[0, late // 16]
-    k[page, late % 16, :, 0] = 1.0
-    v[page, late % 16] = 1.0e37
+    k[page, late % 16, :, 0] = 127 if q8 else 1.0
+    v[page, late % 16] = 127 if q8 else 1.0e37
     q[:] = 0.0
     q[..., 0] = np.linspace(0.0, 7.0 * np.log(2.0), q.shape[1], dtype=np.float32)
     pk.k.copy_(torch.from_numpy(k))
     pk.v.copy_(torch.from_numpy(v))
+    if q8:
+        pk.ks.fill_(1.0 / 127.0)
+        pk.vs.fill_(1.0e37 / 127.0)
     hp, _ = host_pages(pk)
     ref = O.decode_f64(hp, q, tables, kv_len, None, 1.0)
-    for split in (0, 512, 1024):
+    for split in (512, 1024) if q8 and d != 64 else (0, 512, 1024):
         out = pk.decode(dev_f32(q, gpu), dev_i32(tables, gpu), dev_i32(kv_len, gpu), n_heads=2 * rep, max_kv_len=L,
                         scale=1.0, split=split)
         sync()
-        assert rel_err(out, ref).max() < TOL[DTYPE_F32]
+        assert rel_err(out, ref).max() < TOL[dtype]
+
+
+@pytest.mark.parametrize("dtype", [DTYPE_F32, DTYPE_F16, DTYPE_Q8A])
+@pytest.mark.parametrize("step", [-8.1, 0.0, 7.9, 8.0, 8.1])
+@pytest.mark.parametrize("rep", [1, 8])
+def test_running_max_moves_between_pages(gpu, dtype, rep, step):
+    """Scores that move by `step` log2 units from each page of a wave to its
+    next (the four waves take pages in turn), one query head in two holding
+    still: a running max that may lag by 8 units on f16 pages is raised at some
+    of these pages or at none, always for all heads of the group; every page
+    type agrees with the oracle.  Values are exact in f16 and in Q8A codes."""
+    say("running max", DTYPE_NAMES[dtype], rep, step)
+    d, L = 64, 16 * 45 + 5
+    pk, tables, kv_len, q = _case(gpu, dtype, d, rep, 2, (L,), seed=8)
+    k = torch.zeros(pk.k.shape, device=gpu)
+    for p in range((L + 15) // 16):
+        k[int(tables[0, p]), :, :, 0] = p // 4
+    pk.k.copy_(k.to(pk.k.dtype))
+    if dtype == DTYPE_Q8A:
+        pk.ks.fill_(1.0)
+    q[:] = 0.0
+    q[:, ::2, 0] = step * np.log(2.0)
+    hp, _ = host_pages(pk)
+    ref = O.decode_f64(hp, q, tables, kv_len, None, 1.0)
+    for split in (1024, 256):
+        out = pk.decode(dev_f32(q, gpu), dev_i32(tables, gpu), dev_i32(kv_len, gpu), n_heads=2 * rep, max_kv_len=L,
+                        scale=1.0, split=split)
+        sync()
+        assert rel_err(out, ref).max() < TOL[dtype]
 
 
 def test_reference_single_sequence_call_c1_shape(gpu):
