@@ -32,24 +32,22 @@ constexpr float kRescaleSlack = 8.0f;     // log2 units the running max may lag
 // (DATA_FORMAT = 32-bit; no swizzle, no index stride).
 constexpr int kBufferFormat = 0x00020000;
 
-// permlane32_swap(x, x) yields (x[l & ~32], x[l | 32]), permlane16_swap(x, x)
-// yields (x[l & ~16], x[l | 16]): a max or sum of the pair reduces across
-// halves / across adjacent 16-lane rows on the VALU.
+// A max or sum across halves / across adjacent 16-lane rows on the VALU.
 __device__ __forceinline__ float max_xor32(float x) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(int, x), __builtin_bit_cast(int, x), false, false);
-  return fmaxf(__builtin_bit_cast(float, (int)r[0]), __builtin_bit_cast(float, (int)r[1]));
+  const float2 p = swap_xor32(x);
+  return fmaxf(p.x, p.y);
 }
 __device__ __forceinline__ float max_xor16(float x) {
-  const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(int, x), __builtin_bit_cast(int, x), false, false);
-  return fmaxf(__builtin_bit_cast(float, (int)r[0]), __builtin_bit_cast(float, (int)r[1]));
+  const float2 p = swap_xor16(x);
+  return fmaxf(p.x, p.y);
 }
 __device__ __forceinline__ float sum_xor32(float x) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(int, x), __builtin_bit_cast(int, x), false, false);
-  return __builtin_bit_cast(float, (int)r[0]) + __builtin_bit_cast(float, (int)r[1]);
+  const float2 p = swap_xor32(x);
+  return p.x + p.y;
 }
 __device__ __forceinline__ float sum_xor16(float x) {
-  const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(int, x), __builtin_bit_cast(int, x), false, false);
-  return __builtin_bit_cast(float, (int)r[0]) + __builtin_bit_cast(float, (int)r[1]);
+  const float2 p = swap_xor16(x);
+  return p.x + p.y;
 }
 
 __device__ __forceinline__ uint32_t v_swz(int R) { return 2u * (uint32_t)(((R >> 2) & 3) | ((R & 1) << 2)); }
