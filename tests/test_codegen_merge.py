@@ -1,8 +1,8 @@
 """The cross-workgroup merge protocol's code generation (CPU only: hipcc
 cross-compiles gfx950 assembly here).
 
-decode_wg_kernel (partial rows and arrival counts) and q4l_gemv_acc_kernel
-(split partial sums) rely on relaxed agent-scope atomics instead of
+decode_wg_kernel (partial rows and arrival counts), q4l_gemv_acc_kernel and
+q4l_gemm_acc_kernel (split partial sums) rely on relaxed agent-scope atomics instead of
 release/acquire fences, whose agent-scope forms on gfx950 write back or
 invalidate a whole XCD's L2.  That is sound only while the primitives compile
 as checked here, with the library's own device flags: the row stores and loads
