@@ -352,6 +352,7 @@ constexpr int kGemmWaves = 8;
 constexpr int kGemmOut = kGemmVecs * kGemmRows;
 constexpr size_t kGemmPartBytes = kGemmOut * sizeof(float);  // partial sums of one workgroup
 constexpr int kGemmHalf = 128;             // columns staged at once
+constexpr float kGemmMaxScale = 16376.0f;  // the largest f16 below 2^14
 constexpr int kGemmBuf = kGemmVecs * kGemmHalf * 4;  // LDS bytes of one half (hi and lo)
 
 typedef float float16v __attribute__((ext_vector_type(16)));
@@ -482,11 +483,16 @@ __global__ __launch_bounds__(kGemmWaves * kWave) void q4l_gemm_acc_kernel(Q4lArg
     // counts as e = 1) to 13
     const uint32_t mag0 = scr[0] & 0x7FFF7FFFu, mag1 = scr[1] & 0x7FFF7FFFu;
     const uint32_t top = max(max(mag0 & 0xFFFFu, mag0 >> 16), max(mag1 & 0xFFFFu, mag1 >> 16));
-    const int k = 28 - max((int)(top >> 10), 1);
+    // Infinite scales (an effective scale past f16) enter as the largest finite
+    // one, the finite ones beside them as zero, and the half's sum is multiplied
+    // by infinity: as products they would meet x parts and codes of zero.  NaN
+    // scales likewise.
+    const bool nonfinite = top >= 0x7C00u;
+    const int k = nonfinite ? -64 : 28 - max((int)(top >> 10), 1);
     auto weights = [&](int j, int t) {
       const uint32_t sb = scr[j >> 1];
-      const _Float16 s1 =
-          (_Float16)ldexpf((float)__builtin_bit_cast(_Float16, (uint16_t)((j & 1) ? sb >> 16 : sb & 0xFFFFu)), k);
+      const float s0 = (float)__builtin_bit_cast(_Float16, (uint16_t)((j & 1) ? sb >> 16 : sb & 0xFFFFu));
+      const _Float16 s1 = (_Float16)__builtin_amdgcn_fmed3f(ldexpf(s0, k), -kGemmMaxScale, kGemmMaxScale);
       return __builtin_bit_cast(half8, weight_codes_split(wt[j][t])) * half8{s1, s1, s1, s1, s1, s1, s1, s1};
     };
     float16v d[2];
@@ -521,7 +527,7 @@ __global__ __launch_bounds__(kGemmWaves * kWave) void q4l_gemm_acc_kernel(Q4lArg
     }
     stage_w();
     load_w(i + 2);
-    const float back = ldexpf(1.0f, -k);
+    const float back = nonfinite ? (float)__builtin_bit_cast(_Float16, (uint16_t)top) : ldexpf(1.0f, -k);
 #pragma unroll
     for (int v = 0; v < 2; ++v)
 #pragma unroll

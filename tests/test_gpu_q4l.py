@@ -194,6 +194,41 @@ def test_q4l_x_past_f16_range(gpu, n_vec):
     assert np.all(np.abs(yd.cpu().numpy() - ref) <= 2e-6 * (np.abs(x).astype(np.float64) @ wabs.T) + 1e-30)
 
 
+@pytest.mark.parametrize("n_vec", [64, 65])
+def test_q4l_scale_past_f16_range(gpu, n_vec):
+    """Effective scales that overflow f16 (a global scale of 65504 with a local
+    scale above 7) are infinite: where x and the weights of a row are positive
+    its sum is +inf, and -inf with the global scale's sign turned, zero codes,
+    finite sub-blocks of the same row and x that is one f16 (no lo part)
+    notwithstanding, on both sides of the kernels' dividing line; a NaN scale
+    gives NaN; the other rows stay within the bound of
+    test_q4l_gemv_accumulate."""
+    say("q4l infinite scales", n_vec)
+    rng = np.random.default_rng(n_vec)
+    rows, cols = 130, 512
+    disk = _disk(rng, rows, cols).reshape(rows, cols // 256, O.Q4L_DISK_BYTES)
+    disk[:, :, 6:] &= 0x77                                            # positive weights, zero codes among them
+    local = np.array([0x3F, 0x00, 0x70, 0x08], np.uint8)              # sub-blocks 0 and 6 infinite, the others finite
+    for at, g in ((0, 65504.0), (2, -65504.0)):
+        disk[at::9, 1, 0:2] = np.array([g], np.float16).view(np.uint8)
+        disk[at::9, 1, 2:6] = local
+    disk[4::9, 0, 0:2] = np.array([np.nan], np.float16).view(np.uint8)
+    W = Q4LMatrix(disk, rows, cols, gpu)
+    x = rng.uniform(0.5, 2.0, (n_vec, cols)).astype(np.float32)
+    x[::2] = x[::2].astype(np.float16)
+    yd = torch.zeros((n_vec, rows), device=gpu)
+    W.gemv_accumulate(torch.from_numpy(x).to(gpu), yd)
+    sync()
+    got, dev = yd.cpu().numpy(), W.blocks.cpu().numpy()
+    assert int(np.isposinf(got[:, 0::9]).sum()) == got[:, 0::9].size
+    assert int(np.isneginf(got[:, 2::9]).sum()) == got[:, 2::9].size
+    assert int(np.isnan(got[:, 4::9]).sum()) == got[:, 4::9].size
+    rest = np.setdiff1d(np.arange(rows), np.r_[0:rows:9, 2:rows:9, 4:rows:9])
+    with np.errstate(invalid="ignore"):
+        ref = O.q4l_gemv_f64(dev, x, np.zeros((n_vec, rows), np.float32), rows, cols)[:, rest]
+    assert np.all(np.abs(got[:, rest] - ref) <= 2e-6 * ref + 1e-30)
+
+
 def test_q4l_caller_workspace(gpu):
     """A caller's workspace (arrival counts zeroed once) gives the bits of the
     library's buffer, call after call and across shapes that share it (every
