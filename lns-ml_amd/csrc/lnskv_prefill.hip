@@ -132,11 +132,11 @@ constexpr int kPfScaleWave = 512;                                    // K scales
 template <int NH>
 constexpr int kPfQ8Slot = kPfCodeSlot<NH> + 8 * kPfScaleWave;        // codes, then eight waves' scale copies
 
-template <int NH>
+template <int NH, bool UNIFORM>
 __device__ __forceinline__ void pf_issue_q8(const PrefillArgs& a, uint32_t rs, uint32_t kvh, lds_u8* slot,
                                             uint32_t ph0, uint32_t ph1, int w) {
   typedef __attribute__((address_space(3))) void lds_void;
-  w = __builtin_amdgcn_readfirstlane(w);  // as above
+  if constexpr (UNIFORM) w = __builtin_amdgcn_readfirstlane(w);
   const int lane = (int)(threadIdx.x & (kWave - 1));
   const uint32_t page_bytes = kPage * rs;
 #pragma unroll
@@ -618,7 +618,11 @@ __global__ __launch_bounds__((kWave * PfShape<REP, NH>::NW)) void prefill_mfma_k
     const uint32_t bits = (ph0 < a.num_pages ? 1u : 0u) | (ph1 < a.num_pages ? 2u : 0u);
     vbits = (vbits & ~(3u << (2 * sl))) | (bits << (2 * sl));
     if constexpr (Q8)
-      pf_issue_q8<NH>(a, (uint32_t)a.n_kv * (NH * kD), (uint32_t)kvh, ring + sl * kRingSlot, ph0, ph1, w);
+      // uniform w as in pf_issue, except on 128-wide heads with 1 or 2 query
+      // heads, where the other code schedules better (one sequence x 512 tokens
+      // on 2000, 8 kv heads: 132.5 us, 135.9 uniform; 2 heads 184.5 | 187.2;
+      // 4 heads 185.8 both ways; 8 heads 186.5 uniform, 189.8 not)
+      pf_issue_q8<NH, NH == 2 || REP >= 4>(a, (uint32_t)a.n_kv * (NH * kD), (uint32_t)kvh, ring + sl * kRingSlot, ph0, ph1, w);
     else
       pf_issue<Sh::RPW>(a, pl, page_bytes, kvh_off, ring + sl * kSlot, ph0, ph1, w);
   };
