@@ -342,10 +342,11 @@ __global__ __launch_bounds__(kQ4lWaves * kWave) void q4l_gemv_acc_kernel(Q4lArgs
 // issuing the other vector work (a third of it decoding weights) and, of the
 // LDS, ~3000 (each wave reads the half's 32 KiB of x); what hides one behind
 // another is the order below (without the slices, every LDS read waited for
-// right before its product: 10% more time).  4096 x 4096: 46.7 to 51.5 us
-// across boxes at 512 vectors, 21.1 at 128 (135.3 and 34.2 as launches of 64 vectors); 8192 x 8192
-// at 512 vectors 174 (333).  Waves of 64 rows x a quarter block halve the LDS
-// reads but leave no registers for operands read ahead: 15% more time.
+// right before its product: 10% more time).  4096 x 4096: 46.7 to 51.5 us from
+// card to card at 512 vectors, 21.1 at 128 (135.3 and 34.2 as launches of 64
+// vectors); 8192 x 8192 at 512 vectors 174 (333).  Waves of 64 rows x a quarter
+// block halve the LDS reads but leave no registers for operands read ahead: 15%
+// more time.
 constexpr int kGemmVecs = 64;              // vectors per workgroup
 constexpr int kGemmRows = 128;             // weight rows per workgroup
 constexpr int kGemmWaves = 8;
